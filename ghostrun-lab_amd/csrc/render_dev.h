@@ -30,15 +30,39 @@ namespace nd {
 struct RenderScratch {
     uint32_t px[64];          // the line: palette value, 0x40 | backdrop where the background is transparent (in
                               // fast_run, which draws in registers: where the lanes that fetch no sprite store)
-    uint32_t sp[256];         // the sprite line: (7 - rank) << 8 | behind << 7 | palette << 2 | value, 0 = none
-    uint32_t f[36];           // fetches: lo | hi << 8 | attribute << 16; 0-1 carried, 2 + j slot j
-    uint32_t spr[2][8];       // sprite lines: lo | hi << 8 | attr << 16 | x << 24
+    uint32_t sp[256 + 8];     // the sprite line: (7 - rank) << 8 | drawn bits (sprite_bits) | value, 0 = none (the last 8
+                              // words: pixels off the right edge, never read)
+    uint32_t f[36];           // fetches: lo | hi << 8 | attribute (attr_bits); 0-1 carried, 2 + j slot j
+    uint32_t spr[2][8];       // sprite lines: lo | hi << 8 | sprite_bits << 16 | x << 24, lo and hi as drawn (flipped)
     uint32_t pages[34 + 8];   // MMC2: the pages of each slot's fetch, then of each sprite's
     uint4 tab[2];             // the background palette table (bg_table), the latched sprite palette (latch_sprites)
     alignas(16) uint8_t pal[32];
 };
 
 typedef __attribute__((address_space(4))) const uint32_t KU32;
+typedef __attribute__((address_space(1))) uint8_t GlobalU8;
+
+// A value kept in a scalar (vector) register across a loop: VOP3 instructions take no literal, so a constant they use
+// would be moved into a register on every pass, and only one scalar operand, so a second one would be copied.
+__device__ __forceinline__ uint32_t held_s(uint32_t v) {
+    asm volatile("" : "+s"(v));
+    return v;
+}
+__device__ __forceinline__ uint32_t held_v(uint32_t v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+// A tile row's two plane bytes (plane 0 in byte 0, plane 1 in byte 1) with the pixels in the other order.
+__device__ __forceinline__ uint32_t rows_flip(uint32_t x) {
+    return __builtin_amdgcn_perm(__builtin_bitreverse32(x), 0u, 0x0C0C0607u);
+}
+// Where a fetch word holds its 2-bit attribute: bit 0 at bit 2 of byte 2, bit 1 at bit 2 of byte 3, so that a byte
+// permute of two fetch words gives the attribute bits of 4 pixels at the place where the colour lookup needs them
+// (bit 2 of the selector, and the choice of the table's upper half).
+__device__ __forceinline__ uint32_t attr_bits(uint32_t a) { return ((a & 1u) << 18) | ((a & 2u) << 25); }
+// A sprite's entry byte without the pixel's value (OAM attribute byte a): bit 7 set (opaque where the value is not 0),
+// bit 6 in front of the background, bits 2-3 the palette.
+__device__ __forceinline__ uint32_t sprite_bits(uint32_t a) { return 0x80u | ((~a & 0x20u) << 1) | ((a & 3u) << 2); }
 
 // kScalarLog: the frame log was written before this kernel, so its events are read through the scalar cache; else
 // (written earlier in this kernel, by lane 0) by vector loads after the workgroup sync.
@@ -49,6 +73,7 @@ struct RenderSink {
     const uint32_t* log;      // the console's frame log
     const uint8_t *chr_rom, *chr_ram;
     const uint16_t* chr_pairs;   // CHR ROM by tile row (both planes in one word), nullptr with CHR RAM
+    uint32_t flipped;            // chr_pairs' bytes before its second copy, the rows flipped horizontally
     int lane;
     bool mmc2;
     uint32_t ha, hb;          // F indices of the last two fetches
@@ -79,11 +104,9 @@ struct RenderSink {
         const uint32_t k = (uint32_t)lane >> 3, p = (uint32_t)lane & 7u;
         if (k < drawn_n) {
             const uint32_t e = L->spr[drawn][k];
-            const uint32_t attr = (e >> 16) & 0xFFu, b = (attr & 0x40u) ? p : 7u - p;
-            const uint32_t val = ((e >> b) & 1u) | (((e >> (8u + b)) & 1u) << 1);
+            const uint32_t val = ((e >> p) & 1u) | (((e >> (8u + p)) & 1u) << 1);
             const uint32_t x = (e >> 24) + p;
-            if (val && x < 256u)
-                atomicMax(&L->sp[x], ((7u - k) << 8) | ((attr & 0x20u) << 2) | ((attr & 3u) << 2) | val);
+            if (val && x < 256u) atomicMax(&L->sp[x], ((7u - k) << 8) | ((e >> 16) & 0xFFu) | val);
         }
     }
     // A new line (general path): the last two fetches move to F[0], F[1]; nothing drawn yet (0xFF reads as
@@ -108,11 +131,12 @@ struct RenderSink {
         __syncthreads();
     }
     // The two plane bytes of pattern address pa (a row of plane 0; pa + 8 is plane 1) through the packed pages,
-    // plane 0 in the low byte: one 16-bit load with CHR ROM (kPairs), two byte loads with CHR RAM.
+    // plane 0 in the low byte, the leftmost pixel in bit 0: one 16-bit load with CHR ROM (kPairs), two byte loads, flipped,
+    // with CHR RAM.
     template <bool kPairs>
     __device__ uint32_t pattern_of(uint32_t lo, uint32_t hi, uint32_t pa) {
         if constexpr (!kPairs) {
-            return chr_pk(chr_rom, chr_ram, lo, hi, pa) | (chr_pk(chr_rom, chr_ram, lo, hi, pa + 8u) << 8);
+            return rows_flip(chr_pk(chr_rom, chr_ram, lo, hi, pa) | (chr_pk(chr_rom, chr_ram, lo, hi, pa + 8u) << 8));
         } else {
             // the 1 KB slot's page: byte (pa >> 10) & 7 of hi:lo, one byte permute
             const uint32_t page = __builtin_amdgcn_perm(hi, lo, (pa >> 10) & 7u) & 0xFFu;
@@ -134,7 +158,7 @@ struct RenderSink {
         const uint32_t at = ntab[nt_slot(s.nt_map, ntb | 0x3C0u | (col >> 2) | ((v & 0x380u) >> 4))];
         const uint32_t sel = (at >> ((col & 2u) | ((v & 0x40u) >> 4))) & 3u;
         const uint32_t pa = tile * 16u + ((s.ctrl & 0x10u) << 8) + ((v >> 12) & 7u);
-        L->f[j + 2u] = pattern(lo, hi, pa) | (sel << 16);
+        L->f[j + 2u] = pattern(lo, hi, pa) | attr_bits(sel);
     }
     // The background palette as 16 bytes in four words, entry 4a + v: palette a's colour v, and for v = 0 the
     // backdrop with bit 6 set (the transparency mark the sprite priority test reads). Wave-uniform.
@@ -153,26 +177,30 @@ struct RenderSink {
         t[2] = uni(q.z);
         t[3] = uni(q.w);
     }
-    // 4 background pixels, leftmost in the low byte: kk0..kk0 + 3 of the 8 a slot shifts out from fetches p2 (older),
-    // p1 with fine x fx; pixel q is bit 15 - fx - kk0 - q of the two 16-bit plane pairs, with p2's attribute while
-    // fx + kk0 + q < 8, else p1's. All four at once: the planes' 4 bits bit-reversed into place and spread one to a
-    // byte, the attribute chosen per byte by a mask, and the colours looked up 4 at a time by byte permutes of the
-    // palette table.
+    // 4 background pixels, leftmost in the low byte, from the fetch words {hi4:lo4} a byte permute selects from: x = the
+    // two plane pairs of 16 pixels (plane 0 of the older fetch, of the newer one, plane 1 of each, leftmost pixel in the
+    // low bit), shifted by sh (fine x plus the pixel's place in the slot), a1 and a2 the attribute's bits 0 and 1 of each
+    // pixel (attr_bits). The planes' 4 bits are spread one to a byte (a 24-bit multiply, full rate) and the colours looked
+    // up 4 at a time by byte permutes of the palette table t (t0, t2: t[0] and t[2], in vector registers).
+    __device__ uint32_t colours4(uint32_t x, uint32_t sh, uint32_t a1, uint32_t a2, uint32_t t0, uint32_t t1, uint32_t t2,
+                                 uint32_t t3) {
+        const uint32_t lo4 = __builtin_amdgcn_ubfe(x, sh, 4u), hi4 = __builtin_amdgcn_ubfe(x, sh + 16u, 4u);
+        const uint32_t idx = ((lo4 * 0x00204081u) & 0x01010101u) | ((hi4 * 0x00408102u) & 0x02020202u) | a1;
+        const uint32_t lo = __builtin_amdgcn_perm(t1, t0, idx), hi = __builtin_amdgcn_perm(t3, t2, idx);
+        return __builtin_amdgcn_perm(hi, lo, 0x03020100u | a2);   // entries 8..15 from hi
+    }
+    // The same from fetches p2 (older), p1 with fine x fx, pixels kk0..kk0 + 3 of the 8 a slot shifts out: pixel q takes
+    // p2's attribute while fx + kk0 + q < 8, else p1's.
     __device__ uint32_t shift4(uint32_t p2, uint32_t p1, uint32_t kk0, uint32_t fx, const uint32_t t[4]) {
-        const uint32_t sh = fx + kk0;   // 0..11
-        const uint32_t lo16 = ((p2 & 0xFFu) << 8) | (p1 & 0xFFu), hi16 = (p2 & 0xFF00u) | ((p1 >> 8) & 0xFFu);
-        const uint32_t lo4 = __builtin_bitreverse32(lo16 << (16u + sh)) & 0xFu;   // pixel q at bit q
-        const uint32_t hi4 = __builtin_bitreverse32(hi16 << (16u + sh)) & 0xFu;
-        const uint32_t val = ((lo4 * 0x00204081u) & 0x01010101u) | (((hi4 * 0x00204081u) & 0x01010101u) << 1);
-        const int32_t b = 8 - (int32_t)sh;   // pixels q < b take p2's attribute
+        const uint32_t sh = fx + kk0, sa = attr_sel(sh, 0x02020202u);   // sh: 0..11
+        return colours4(__builtin_amdgcn_perm(p1, p2, 0x05010400u), sh, __builtin_amdgcn_perm(p1, p2, sa),
+                        __builtin_amdgcn_perm(p1, p2, sa + 0x01010101u), t[0], t[1], t[2], t[3]);
+    }
+    // The byte selector of pixels q = 0..3's attribute byte: base where sh + q < 8, else base ^ 4 (the other fetch).
+    __device__ uint32_t attr_sel(uint32_t sh, uint32_t base) {
+        const int32_t b = 8 - (int32_t)sh;   // pixels q < b take the older fetch's
         const uint32_t m = b >= 4 ? 0xFFFFFFFFu : b <= 0 ? 0u : (1u << (8 * b)) - 1u;
-        // (byte selects by v_perm_b32, whose selector byte k picks byte k of {src0:src1}, src1 the low four: full
-        // rate, where spreading a byte by a 32-bit multiply is a quarter-rate instruction)
-        const uint32_t attr = __builtin_amdgcn_perm((p1 >> 16) & 3u, (p2 >> 16) & 3u, ~m & 0x04040404u);
-        const uint32_t idx = (attr << 2) | val;   // palette entry per byte, 0..15
-        const uint32_t sel = idx & 0x07070707u;
-        const uint32_t lo = __builtin_amdgcn_perm(t[1], t[0], sel), hi = __builtin_amdgcn_perm(t[3], t[2], sel);
-        return __builtin_amdgcn_perm(hi, lo, 0x03020100u | ((idx >> 1) & 0x04040404u));   // entries 8..15 from hi
+        return base ^ (~m & 0x04040404u);
     }
     __device__ void on_run(const Rs& s, int32_t first, int32_t last, int32_t out, bool pixels) {
         __syncthreads();   // the walker's page and palette writes
@@ -243,11 +271,15 @@ struct RenderSink {
             const uint32_t pa = (base + (flip & (7u + ((ctrl & 0x20u) >> 1))) + ((r2 ^ flip) - flip)) & 0x1FFFu;
             const uint32_t pk = mmc2 ? L->pages[34 + rank] : 0u;
             const uint32_t lo = mmc2 ? pk : s.chr_lo, hi = mmc2 ? pk : s.chr_hi;
-            L->spr[target][rank] = pattern(lo, hi, pa) | (e & 0xFFFF0000u);
+            const uint32_t pix = pattern(lo, hi, pa);
+            L->spr[target][rank] = ((e & 0x400000u) ? rows_flip(pix) : pix) | (sprite_bits((e >> 16) & 0xFFu) << 16) |
+                                   (e & 0xFF000000u);
         }
         fetched = target;
         return sel;
     }
+    // The opaque pixels of a sprite line's entry, leftmost in bit 7 (the entry is flipped as drawn: no flip is left to do).
+    __device__ uint32_t first_bits(uint32_t e) { return __builtin_bitreverse32((e & 0xFFu) | ((e >> 8) & 0xFFu)) >> 24; }
     // What RefreshSprites needs of the fetch (after the sync).
     __device__ void sprite_fetch_done(Rs& s, uint64_t sel) {
         const uint32_t n = (uint32_t)__builtin_popcountll(sel);
@@ -255,8 +287,8 @@ struct RenderSink {
         s.f_blurp = (uint32_t)(sel & 1u);
         if (s.f_n) {
             const uint32_t e0 = uni(L->spr[fetched][0]);
-            s.f_bits = (e0 & 0xFFu) | ((e0 >> 8) & 0xFFu);
-            s.f_attr = (e0 >> 16) & 0xFFu;
+            s.f_bits = first_bits(e0);
+            s.f_attr = 0;
             s.f_x = e0 >> 24;
         }
     }
@@ -289,6 +321,20 @@ struct RenderSink {
         t[2] = uni(q.z);
         t[3] = uni(q.w);
     }
+    // Four sprite line entries over the background pixels w, one per byte: a sprite pixel (bit 7) shows in front (bit
+    // 6), or behind a transparent background pixel (w's bit 6, the backdrop mark), where `shown` has bit 6 set (not in
+    // the left 8 with sprite clipping); its colour from the latched sprite palette (s0..s3, s0 and s2 in vector registers)
+    // by byte permutes (entry = palette << 2 | value). id, c04, c07, p01, p23: kId ... kP23, held in registers or not.
+    static constexpr uint32_t kId = 0x03020100u, kC04 = 0x04040404u, kC07 = 0x07070707u, kP01 = 0x0C0C0400u, kP23 = 0x04000C0Cu;
+    __device__ uint32_t sprites4(const uint4& sp, uint32_t w, uint32_t shown, uint32_t s0, uint32_t s1, uint32_t s2,
+                                 uint32_t s3, uint32_t id, uint32_t c04, uint32_t c07, uint32_t p01, uint32_t p23) {
+        const uint32_t eb = __builtin_amdgcn_perm(sp.y, sp.x, p01) | __builtin_amdgcn_perm(sp.w, sp.z, p23);
+        const uint32_t eb1 = eb >> 1, show = ((eb1 & w) | eb) & shown;
+        const uint32_t sel = eb & c07;
+        const uint32_t lo = __builtin_amdgcn_perm(s1, s0, sel), hi = __builtin_amdgcn_perm(s3, s2, sel);
+        const uint32_t col = __builtin_amdgcn_perm(hi, lo, (eb1 & c04) | id);
+        return __builtin_amdgcn_perm(col, w, id | (show >> 4));   // the shown bytes from col
+    }
     // spt: the latched sprite palette (sprite_table). The line's emphasis is the caller's (the mask at this point).
     __device__ void compose(Rs& s, int32_t l, uint32_t w, uint8_t* obs, const uint32_t spt[4]) {
         const bool expanded = s.spork != 0, sprites = (s.mask & 0x10u) && expanded;
@@ -298,18 +344,9 @@ struct RenderSink {
             const uint4 sp = reinterpret_cast<const uint4*>(L->sp)[lane];
             reinterpret_cast<uint4*>(L->sp)[lane] = make_uint4(0u, 0u, 0u, 0u);
             if (sprites) {
-                // the four pixels at once, one per byte: a sprite pixel (value != 0) shows in front, or behind a
-                // transparent background pixel (bit 6, the backdrop mark), except in the left 8 with sprite
-                // clipping; its colour from the latched sprite palette by byte permutes (entry = palette << 2 | value)
-                const uint32_t eb = (sp.x & 0xFFu) | ((sp.y & 0xFFu) << 8) | ((sp.z & 0xFFu) << 16) | (sp.w << 24);
-                const uint32_t opaque = (eb | (eb >> 1)) & 0x01010101u;
-                const uint32_t front = ~(eb >> 7) & 0x01010101u, clear_bg = (w >> 6) & 0x01010101u;
                 const bool clipped = !(s.mask & 0x04u) && lane < 2;
-                const uint32_t show = clipped ? 0u : opaque & (front | clear_bg);
-                const uint32_t sel = eb & 0x07070707u;
-                const uint32_t lo = __builtin_amdgcn_perm(spt[1], spt[0], sel), hi = __builtin_amdgcn_perm(spt[3], spt[2], sel);
-                const uint32_t col = __builtin_amdgcn_perm(hi, lo, 0x03020100u | ((eb >> 1) & 0x04040404u));
-                w = __builtin_amdgcn_perm(col, w, 0x03020100u | (show << 2));   // the shown bytes from col
+                w = sprites4(sp, w, clipped ? 0u : 0x40404040u, spt[0], spt[1], spt[2], spt[3], kId, kC04, kC07,
+                             kP01, kP23);
             }
         }
         if (l < 8) return;
@@ -357,9 +394,19 @@ struct RenderSink {
     //     and masks rather than lane-divergent branches: the CU's scalar unit is what the emulator's waves need.
     // With rendering off the lines are the backdrop: nothing is fetched, v stays, no sprite is drawn and no sprite-0
     // check can hit (the backdrop is transparent).
+    // The loop is bound by vector issue (a wave's share of it also delays the emulator's waves beside it), so everything
+    // that can be laid out ahead is: CHR rows with the leftmost pixel in bit 0 (a pixel's 4 bits are one v_bfe, no bit
+    // reversal) and a second copy flipped horizontally (a flipped entry reads the other copy, no select per pixel), the
+    // attribute and the sprite's priority and palette at the bits the byte permutes take, each lane's selectors for the
+    // run, 32-bit offsets from scalar bases, and constants in registers. 66 vector and 28 scalar instructions a line by
+    // the counters (8192 console-frames of the NROM cart) where the plain formulation took 101 and 33; a decision of 8192
+    // NROM consoles 2.87 -> 2.66 ms, of 16384 MMC3 consoles 10.3 -> 9.9 ms.
     // kSpr: sprites on (mask bit 4) for the run.
     template <bool kPairs, bool kSpr>
     __device__ void fast_run(Rs& s, int32_t l, int32_t stop, uint8_t* obs, uint8_t* emph) {
+        // (opaque: what follows from the lane is worked out in each run, not held through the frame in vector registers)
+        int lane = this->lane;
+        asm volatile("" : "+v"(lane));
         uint32_t t[4];
         bg_table(t);
         const uint32_t back4 = (t[0] & 0xFFu) * 0x01010101u;
@@ -381,12 +428,23 @@ struct RenderSink {
         const uint32_t flip = (uint32_t)((int32_t)(e << 8) >> 31);
         const uint32_t sb = (h == 16u ? ((st & 1u) << 12) + ((st & 0xFEu) << 4) : (st << 4) + table8) +
                             (flip & (7u + ((ctrl & 0x20u) >> 1)));
-        const uint32_t slot = ((uint32_t)lane + 1u) >> 1, kk0 = ((uint32_t)lane & 1u) * 4u;
-        // (kPairs) the entry's rows in one 1 KB page: row r's pair at sp_i0 + r, or flipped sp_i0 + h - 1 - r. With
-        // pb its row 0's pattern address (16-aligned, 32 for 8x16), the pattern of row r is at pb + r for 8x8, pb + r
-        // + (r & 8) for 8x16 (the tile after), whose pair index is that of pb plus r; flipped the rows run backwards.
-        const uint32_t sp_i0 = kPairs ? pairs_index(s.chr_lo, s.chr_hi, sb - (flip & (7u + ((ctrl & 0x20u) >> 1)))) +
-                                            (flip & (h - 1u))
+        // what the entry's line holds besides its pixels
+        const uint32_t e_bits = held_v((sprite_bits((e >> 16) & 0xFFu) << 16) | (e & 0xFF000000u)), e_y = e & 0xFFu;
+        const uint32_t slot = ((uint32_t)lane + 1u) >> 1, sh = s.fx + ((uint32_t)lane & 1u) * 4u;
+        // the byte selectors of this lane's 16 pixels and of their attributes from {the other lane's fetch : its own}:
+        // the older fetch is its own on even lanes, the other's on odd ones
+        const uint32_t own = (lane & 1) ? 4u : 0u;
+        // (lanes without background select zeros: entry 0 of palette 0, the backdrop)
+        const uint32_t x_sel = bg_on ? 0x05010400u ^ (own * 0x01010101u) : 0x0C0C0C0Cu;
+        const uint32_t a_sel = bg_on ? attr_sel(sh, 0x02020202u ^ (own * 0x01010101u)) : 0x0C0C0C0Cu;
+        const uint32_t a_sel2 = bg_on ? a_sel + 0x01010101u : 0x0C0C0C0Cu;
+        // (kPairs) the entry's rows in one 1 KB page: row r's pair is at byte sp_b0 + 2 r, or vertically
+        // flipped sp_b0 - 2 r. With pb its row 0's
+        // pattern address (16-aligned, 32 for 8x16), the pattern of row r is at pb + r for 8x8, pb + r + (r & 8) for 8x16
+        // (the tile after), whose pair index is that of pb plus r; vertically flipped the rows run backwards, horizontally
+        // flipped they are those of the table's second copy.
+        const uint32_t sp_b0 = kPairs ? 2u * (pairs_index(s.chr_lo, s.chr_hi, sb - (flip & (7u + ((ctrl & 0x20u) >> 1)))) +
+                                              (flip & (h - 1u))) + ((e & 0x400000u) ? flipped : 0u) - flip
                                       : 0u;
         // the latched sprite palette. With sprites on, the line before the run ended with RefreshSprites: it latched
         // the palette as it is now, or latched nothing (no sprite is drawn before a latch in the run, which takes this
@@ -395,18 +453,25 @@ struct RenderSink {
         if (spr_on && sp_stale) latch_table();
         uint32_t spt[4];
         sprite_table(spt);
-        // what else the run holds fixed: greyscale (rendering is on), the left-8 sprite clip, t's horizontal bits
+        // what else the run holds fixed: greyscale (rendering is on), the left-8 sprite clip, t's horizontal bits, the
+        // colour tables' words that share a permute with another scalar, the permutes' constants
         const uint32_t keep4 = (mask & 0x01u) ? 0x30303030u : 0x3F3F3F3Fu;
-        const uint32_t show_m = !(mask & 0x04u) && lane < 2 ? 0u : 0xFFFFFFFFu;
+        const uint32_t shown = !(mask & 0x04u) && lane < 2 ? 0u : 0x40404040u;
         const uint32_t t_h = s.t & 0x041Fu, kk = (uint32_t)lane >> 3, px = (uint32_t)lane & 7u;
+        const uint32_t t0 = held_v(t[0]), t2 = held_v(t[2]);
+        const uint32_t s0 = kSpr ? held_v(spt[0]) : 0u, s2 = kSpr ? held_v(spt[2]) : 0u;
+        const uint32_t id = kSpr ? held_v(kId) : 0u, c04 = kSpr ? held_s(kC04) : 0u, c07 = kSpr ? held_s(kC07) : 0u;
+        const uint32_t p01 = kSpr ? held_s(kP01) : 0u, p23 = kSpr ? held_s(kP23) : 0u;
+        const uint32_t rank_bits = (7u - kk) << 8;
         // the row's 60 words are stored by all 64 lanes: lanes 0 and 1 store lane 2's word, 62 and 63 lane 61's
-        const int32_t ox = 4 * (lane < 2 ? 0 : lane > 61 ? 59 : lane - 2);
+        const uint32_t ox = 4u * (uint32_t)(lane < 2 ? 0 : lane > 61 ? 59 : lane - 2);
+        GlobalU8* row_at = (GlobalU8*)obs + (ptrdiff_t)(l - 8) * RLE_OBS_W;
         // The run's state in registers, written back after it. The two sprite buffers are 0 and 1, so the one a
-        // fetch fills (the one not latched) is drawn ^ 1. spork: a line was latched at the end of the line before
-        // (with sprites on the only way it is set in the run; with sprites off nothing is drawn, so the latched line
-        // is not expanded: the sprite line stays clear, as the compose would leave it).
-        uint32_t vl = s.v, dr = drawn, dr_n = drawn_n, spork = s.spork, tgt = drawn ^ 1u;
-        uint32_t hit = s.hit, sp_bits = s.sphit_bits, f_bits = s.f_bits, f_attr = s.f_attr, f_x = s.f_x;
+        // fetch fills (the one not latched) is drawn ^ 1. With sprites on, dr_n is 0 where no line was latched at the end
+        // of the line before (spork; the only way it is set in the run); with sprites off nothing is drawn, so the
+        // latched line is not expanded: the sprite line stays clear, as the compose would leave it.
+        uint32_t vl = s.v, dr = drawn, dr_n = kSpr && !s.spork ? 0u : drawn_n, tgt = drawn ^ 1u;
+        uint32_t hit = s.hit, sp_bits = s.sphit_bits, f_bits = s.f_bits, f_x = s.f_x;
         int32_t sphitx = s.sphitx, hit_x = s.hit_x;
         uint64_t sel = 0;
         uint32_t key = 0xFFFFFFFFu, tb = 0, tsel = 0, vline = vl;
@@ -419,33 +484,39 @@ struct RenderSink {
                 const uint32_t ntb = 0x2000u | (vs & 0x0C00u), col = vs & 31u;
                 const uint32_t tile = ntab[nt_slot(s.nt_map, ntb | (vs & 0x3FFu))];
                 const uint32_t at = ntab[nt_slot(s.nt_map, ntb | 0x3C0u | (col >> 2) | ((vs & 0x380u) >> 4))];
-                tsel = ((at >> ((col & 2u) | ((vs & 0x40u) >> 4))) & 3u) << 16;
+                tsel = attr_bits((at >> ((col & 2u) | ((vs & 0x40u) >> 4))) & 3u);
                 tb = tile * 16u + ptab;
-                if constexpr (kPairs) tb = pairs_index(s.chr_lo, s.chr_hi, tb);   // (fine y adds to the index)
+                if constexpr (kPairs) tb = 2u * pairs_index(s.chr_lo, s.chr_hi, tb);   // (fine y adds 2 bytes a row)
             }
             // FetchSpriteData for line l + 1 into buffer tgt (every lane fetches its entry's row, only the first eight
             // on the line keep it)
-            const uint32_t row = (uint32_t)(l - (int32_t)(e & 0xFFu));
-            sel = __ballot(row < h);
-            const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(sel >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)sel, 0u));
-            uint32_t spp;
+            const uint32_t row = (uint32_t)l - e_y;
+            const bool in = row < h;
+            sel = __ballot(in);
+            // the entry's place among those on the line, at 8 or above for an entry off it
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(sel >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)sel, in ? 0u : 8u));
+            uint32_t spp, mine;
+            const uint8_t* const pairs = reinterpret_cast<const uint8_t*>(chr_pairs);
             if constexpr (kPairs) {
-                const uint32_t rc = row < h ? row : 0u;   // (an entry off the line reads its row 0: in bounds)
-                spp = chr_pairs[sp_i0 + ((rc ^ flip) - flip)];
+                // (an entry off the line reads its row 0: in bounds)
+                spp = *reinterpret_cast<const uint16_t*>(pairs + ((((in ? row : 0u) << 1) ^ flip) + sp_b0));
+                mine = *reinterpret_cast<const uint16_t*>(pairs + (tb + ((vl >> 11) & 14u)));
             } else {
                 const uint32_t r2 = row + (row & 8u);
                 spp = pattern_of<kPairs>(s.chr_lo, s.chr_hi, (sb + ((r2 ^ flip) - flip)) & 0x1FFFu);
+                if (e & 0x400000u) spp = rows_flip(spp);
+                mine = pattern_of<kPairs>(s.chr_lo, s.chr_hi, tb + ((vl >> 12) & 7u));
             }
-            const uint32_t sp = spp | (e & 0xFFFF0000u);
-            const uint32_t mine = (kPairs ? (uint32_t)chr_pairs[tb + ((vl >> 12) & 7u)]
-                                          : pattern_of<kPairs>(s.chr_lo, s.chr_hi, tb + ((vl >> 12) & 7u))) | tsel;
+            const uint32_t sp = spp | e_bits;
+            mine |= tsel;
             const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)mine, 0xB1, 0xF, 0xF, false);   // lane ^ 1
             // (the lanes that keep nothing store into their own word of the line buffer, unused by this path)
-            const uint32_t slot_k = rank + (row < h ? 0u : 8u);
-            *(slot_k < 8u ? &L->spr[tgt][slot_k] : &L->px[lane]) = sp;
+            *(rank < 8u ? &L->spr[tgt][rank] : &L->px[lane]) = sp;
             const uint32_t fetched_now = tgt;
-            const uint32_t bgw = shift4(lane & 1 ? other : mine, lane & 1 ? mine : other, kk0, s.fx, t);
-            uint32_t w = bg_on ? bgw : back4;
+            uint32_t w = colours4(__builtin_amdgcn_perm(other, mine, x_sel), sh,
+                                  __builtin_amdgcn_perm(other, mine, a_sel), __builtin_amdgcn_perm(other, mine, a_sel2), t0,
+                                  t[1], t2, t[3]);
             if (sphitx != kNoCheck) {   // (check_hit on the run's registers: the background pixels)
                 const int32_t end = sphitx + 8 < 255 ? sphitx + 8 : 255;
                 uint32_t first = 4u;
@@ -462,36 +533,28 @@ struct RenderSink {
                     hit_x = 4 * ln + __builtin_amdgcn_readlane((int)first, ln);
                 }
             }
-            if (spr_on && spork) {
+            if (kSpr && dr_n) {
                 // this line's sprites: lane 8k + p expands pixel p of latched sprite k (expand_sprites), every lane
                 // issuing its LDS max, a zero (no change) where there is nothing to draw
-                const uint32_t es = L->spr[dr][kk];
-                const uint32_t attr = (es >> 16) & 0xFFu, b = (attr & 0x40u) ? px : 7u - px;
-                const uint32_t x = (es >> 24) + px;
-                uint32_t val = ((es >> b) & 1u) | (((es >> (8u + b)) & 1u) << 1);
-                // (k < drawn_n and x < 256 as sign masks)
-                val &= (uint32_t)((int32_t)(x - 256u) >> 31) & (uint32_t)((int32_t)(kk - dr_n) >> 31);
-                const uint32_t ent = ((7u - kk) << 8) | ((attr & 0x20u) << 2) | ((attr & 3u) << 2) | val;
-                atomicMax(&L->sp[x & 0xFFu], ent & (0u - (val < 1u ? val : 1u)));
+                uint32_t es = L->spr[dr][kk];
+                es = kk < dr_n ? es : 0u;
+                const uint32_t val = __builtin_amdgcn_ubfe(es, px, 1u) | (__builtin_amdgcn_ubfe(es, px + 8u, 1u) << 1);
+                const uint32_t ent = rank_bits | ((es >> 16) & 0xFFu) | val;
+                atomicMax(&L->sp[(es >> 24) + px], val != 0u ? ent : 0u);
                 __syncthreads();
                 // compose: the sprite pixels over the background, the lane's part of L->sp cleared
                 const uint4 spq = reinterpret_cast<const uint4*>(L->sp)[lane];
                 reinterpret_cast<uint4*>(L->sp)[lane] = make_uint4(0u, 0u, 0u, 0u);
-                const uint32_t eb = (spq.x & 0xFFu) | ((spq.y & 0xFFu) << 8) | ((spq.z & 0xFFu) << 16) | (spq.w << 24);
-                const uint32_t opaque = (eb | (eb >> 1)) & 0x01010101u;
-                const uint32_t front = ~(eb >> 7) & 0x01010101u, clear_bg = (w >> 6) & 0x01010101u;
-                const uint32_t show = opaque & (front | clear_bg) & show_m;
-                const uint32_t ssel = eb & 0x07070707u;
-                const uint32_t lo = __builtin_amdgcn_perm(spt[1], spt[0], ssel), hi = __builtin_amdgcn_perm(spt[3], spt[2], ssel);
-                const uint32_t col = __builtin_amdgcn_perm(hi, lo, 0x03020100u | ((eb >> 1) & 0x04040404u));
-                w = __builtin_amdgcn_perm(col, w, 0x03020100u | (show << 2));
+                w = sprites4(spq, w, shown, s0, spt[1], s2, spt[3], id, c04, c07, p01, p23);
             }
+            asm volatile("" : "+s"(row_at));   // (a scalar base: the lane's offset is 32 bits)
             if (l >= 8) {
                 uint32_t wo = w & keep4;
                 wo = (uint32_t)__builtin_amdgcn_update_dpp((int)wo, (int)wo, 0xEA, 0x1, 0x1, false);   // 0-3: [2,2,2,3]
                 wo = (uint32_t)__builtin_amdgcn_update_dpp((int)wo, (int)wo, 0x54, 0x8, 0x8, false);   // 60-63: [0,1,1,1]
-                *reinterpret_cast<uint32_t*>(obs + (l - 8) * RLE_OBS_W + ox) = wo;
+                *(__attribute__((address_space(1))) uint32_t*)(row_at + ox) = wo;
             }
+            row_at += RLE_OBS_W;
             // the end of the line: Fixit1 and Fixit2 (v from t horizontally), RefreshSprites
             sphitx = kNoCheck;
             if (__builtin_expect((vl & 0x7000u) == 0x7000u, 0)) vl = y_step(vl);
@@ -499,18 +562,16 @@ struct RenderSink {
             vl = (vl & 0x7BE0u) | t_h;
             if (spr_on) {
                 const uint32_t n = (uint32_t)__builtin_popcountll(sel);
-                spork = n < 1u ? n : 1u;
-                dr_n = spork ? (n < 8u ? n : 8u) : dr_n;
-                dr = spork ? fetched_now : dr;
+                dr_n = n < 8u ? n : 8u;
+                dr = n ? fetched_now : dr;
             }
             if (__builtin_expect((uint32_t)sel & 1u, 0)) {   // sprite 0 fetched for the next line: what RefreshSprites keeps
                 const uint32_t e0 = (uint32_t)__builtin_amdgcn_readlane((int)sp, 0);
-                f_bits = (e0 & 0xFFu) | ((e0 >> 8) & 0xFFu);
-                f_attr = (e0 >> 16) & 0xFFu;
+                f_bits = first_bits(e0);
                 f_x = e0 >> 24;
                 if (spr_on && !hit && f_bits) {
                     sphitx = (int32_t)f_x;
-                    sp_bits = (f_attr & 0x40u) ? __builtin_bitreverse32(f_bits) >> 24 : f_bits;
+                    sp_bits = f_bits;
                 }
             }
             tgt = dr ^ 1u;
@@ -523,9 +584,9 @@ struct RenderSink {
         s.f_n = n_last < 8u ? n_last : 8u;
         s.f_blurp = (uint32_t)(sel & 1u);
         s.f_bits = f_bits;
-        s.f_attr = f_attr;
+        s.f_attr = 0;
         s.f_x = f_x;
-        s.spork = spork;
+        if (kSpr) s.spork = dr_n ? 1u : 0u;
         s.hit = hit;
         s.hit_x = hit_x;
         s.sphitx = sphitx;
@@ -554,7 +615,7 @@ __device__ __forceinline__ void draw_frame(RenderScratch* L, uint8_t* nt, uint8_
     reinterpret_cast<uint4*>(L->sp)[lane] = make_uint4(0u, 0u, 0u, 0u);
     __syncthreads();
     const bool mmc2 = cart.board == NES_BOARD_MMC2;
-    RenderSink<kScalarLog> sink{L, nt, oam, log, cart.chr, chr_ram, cart.chr_pairs, lane, mmc2, 0u, 1u, 0u, 0u, 0u,
+    RenderSink<kScalarLog> sink{L, nt, oam, log, cart.chr, chr_ram, cart.chr_pairs, cart.chr_pages1 * 1024u, lane, mmc2, 0u, 1u, 0u, 0u, 0u,
                                 true, true};
     Rs s;
     rs_load(s, sink, log, uni(log_n), mmc2 ? cart.chr_pages1 : 0u);

@@ -1354,12 +1354,22 @@ void* rlenv_create(int ngames, const int* game_ids, const uint8_t* const* roms, 
             if (!p.chr.empty()) {
                 chr = static_cast<uint8_t*>(env->mem.alloc(p.chr.size()));
                 env->mem.upload(chr, p.chr.data(), p.chr.size());
-                std::vector<uint16_t> pairs(p.chr.size() / 2);   // per 16-byte tile: row r = plane 0 | plane 1 << 8
+                // per 16-byte tile: row r = plane 0 | plane 1 << 8, the leftmost pixel in bit 0; then all rows again
+                // flipped horizontally (as the cartridge holds them)
+                const auto left_first = [](uint8_t b) {
+                    b = (uint8_t)((b >> 4) | (b << 4));
+                    b = (uint8_t)(((b & 0xCCu) >> 2) | ((b & 0x33u) << 2));
+                    return (uint8_t)(((b & 0xAAu) >> 1) | ((b & 0x55u) << 1));
+                };
+                std::vector<uint16_t> pairs(p.chr.size());
                 for (size_t t = 0; t < p.chr.size(); t += 16)
-                    for (size_t r = 0; r < 8; ++r)
-                        pairs[t / 2 + r] = (uint16_t)(p.chr[t + r] | (p.chr[t + 8 + r] << 8));
-                chr_pairs = static_cast<uint16_t*>(env->mem.alloc(p.chr.size()));
-                env->mem.upload(chr_pairs, pairs.data(), p.chr.size());
+                    for (size_t r = 0; r < 8; ++r) {
+                        const uint8_t lo = p.chr[t + r], hi = p.chr[t + 8 + r];
+                        pairs[t / 2 + r] = (uint16_t)(left_first(lo) | (left_first(hi) << 8));
+                        pairs[p.chr.size() / 2 + t / 2 + r] = (uint16_t)(lo | (hi << 8));
+                    }
+                chr_pairs = static_cast<uint16_t*>(env->mem.alloc(pairs.size() * 2));
+                env->mem.upload(chr_pairs, pairs.data(), pairs.size() * 2);
             }
             uint32_t chr_pages = p.chr.empty() ? 8u : (uint32_t)(p.chr.size() / 1024u);
             if (chr_pages & (chr_pages - 1u)) throw std::runtime_error("CHR size must be a power of two");
