@@ -95,8 +95,19 @@ RL10G_FN int rl10_keyset_insert(uint32_t* slots, uint32_t cap, uint32_t* count, 
     return -1;
 }
 
+/* On the device the lanes of a wave that call this all hold the same key set (lane 0 alone in a decision's finish, the
+ * 64 lanes of the env's wave in rl10_run), and share the stores; the fence keeps a lane's later probes of slots that
+ * another lane cleared behind those stores. */
 RL10G_FN void rl10_keyset_clear(uint32_t* slots, uint32_t cap) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const uint64_t on = __builtin_amdgcn_ballot_w64(true);
+    const uint32_t first = __builtin_amdgcn_mbcnt_hi((uint32_t)(on >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)on, 0u));
+    const uint32_t step = (uint32_t)__builtin_popcountll(on);
+    for (uint32_t i = first; i < cap; i += step) slots[i] = 0u;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#else
     for (uint32_t i = 0; i < cap; ++i) slots[i] = 0u;
+#endif
 }
 
 /* ------------------------------------------------------------------------------------------------ helpers */
@@ -650,6 +661,25 @@ RL10G_FN Rl10Signals rl10_punchout(const uint8_t* r, Rl10Reader* e) {
     s.game_over = (uint8_t)(loss || rl10_u8(r, 0x172) * 10 + rl10_u8(r, 0x173) > 0);
     s.won = (uint8_t)(winst && fight == 13);
     return s;
+}
+
+/* The 128-byte lines of the 2 KB RAM (bit l: addresses 128 l .. 128 l + 127) that a game's reader reads: at most 5 of
+ * the 16, so that rl10_run moves 128 to 640 bytes of an env-step's 2048. */
+RL10G_HD uint32_t rl10_ram_lines(int game) {
+    switch (game) {
+        case RL10_SMB: return 1u << 0 | 1u << 1 | 1u << 14 | 1u << 15;
+        case RL10_PACMAN: return 1u << 0;
+        case RL10_EXCITEBIKE: return 1u << 0 | 1u << 1 | 1u << 7;
+        case RL10_CONTRA: return 1u << 0 | 1u << 1 | 1u << 10 | 1u << 11 | 1u << 15;
+        case RL10_CASTLEVANIA: return 1u << 0 | 1u << 3 | 1u << 8 | 1u << 15;
+        case RL10_GRADIUS: return 1u << 0 | 1u << 15;
+        case RL10_ZELDA: return 1u << 0 | 1u << 1 | 1u << 12;
+        case RL10_TETRIS: return 1u << 0 | 1u << 1;
+        case RL10_TECMOBOWL: return 1u << 0 | 1u << 1;
+        case RL10_KAGE: return 1u << 0 | 1u << 1 | 1u << 13 | 1u << 14 | 1u << 15;
+        case RL10_FINALMISSION: return 1u << 0 | 1u << 1 | 1u << 9;
+        default: return 1u << 0 | 1u << 2 | 1u << 6 | 1u << 7;   /* Punch-Out */
+    }
 }
 
 /* The signals of a game other than SMB from its 2 KB RAM (reward10.cuh:509-524). t: the tracker (its overflow flag),

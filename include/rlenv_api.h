@@ -157,7 +157,7 @@ int rlenv_jit_check(const char* code, size_t size, int32_t* out, char* where, si
 int rl10_smb_run(const uint8_t* ram15, int T, int N, int frames, void* state, float* reward, uint8_t* done,
                  void* stream);
 
-/* The reward10 tracker of any game (ids as in rlenv_create) on device RAM: T steps of N envs, one env per thread.
+/* The reward10 tracker of any game (ids as in rlenv_create) on device RAM: T steps of N envs, one env per wave.
  * ram: u8 [T, N, 2048] device, the 2 KB RAM of each env-step; frames: i32 [T, N] emulated frames per step;
  * state: Rl10State [N], reader: Rl10Reader [N] (include/rlenv_state.h) and keys: u32 [N * cap], cap =
  * rl10_keyset_capacity(game) (include/rl10_games.h; keys may be null when it is 0), all zeroed for a fresh env and

@@ -10,14 +10,14 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import GOLDEN, HIP_LIB
+from helpers import GOLDEN, HIP_LIB, ORACLE_LIB
 from rl import synth
 from rl.rlenv import GAMES, RlEnv
 from test_env_games import KEY_CAP, all_games, roms
 from test_gpu_parity import OUTS
 
 sys.path.insert(0, str(Path(__file__).resolve().parent / 'golden'))
-from reward10_ram import trajectory  # noqa: E402
+from reward10_ram import SPECS, trajectory  # noqa: E402
 
 FIX = np.load(GOLDEN / 'reward10_games.npz')
 
@@ -136,3 +136,45 @@ def test_all_games_env_parity_with_level_starts_and_places():
     assert np.array_equal(cpu.state_dict()['env'], gpu.state_dict()['env'])
     assert run_pair(cpu, gpu, 20, g) > 0, 'no episode started from a saved slot'
     assert np.array_equal(cpu.state_dict()['env'], gpu.state_dict()['env'])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('T,N', [(1, 1), (4, 3), (5, 33), (3, 97), (9, 130)])
+def test_rl10_run_ragged_sizes_and_split_calls_match_the_oracle(T, N):
+    """rl10_run at the edges of its waves a workgroup (4) and rows a load (4), from RAM at an odd address, with fresh
+    random RAM on every step in what the reader does not read: outputs, tracker, reader state and key sets of every
+    game equal the oracle's bit for bit after two calls in a row."""
+    print(f'case: rl10_run on the GPU, every game, two calls of T={T} N={N}', flush=True)
+    libs = {'cpu': ctypes.CDLL(str(ORACLE_LIB)), 'cuda': hip()}
+    libs['cpu'].rl10_run.argtypes = libs['cuda'].rl10_run.argtypes
+    rng = np.random.default_rng(T * 1000 + N)
+    for gi, game in enumerate(GAMES):
+        cap = KEY_CAP.get(game, 0)
+        if gi == 0:
+            smb = synth.smb_ram15(5, N, 2 * T)
+            ram = synth.expand_ram(smb)
+            read = list(synth.SMB_ADDRS)
+        else:
+            ram = np.stack([trajectory(game, 100 + e, 2 * T)[0] for e in range(N)], 1)
+            read = sorted(SPECS[game])
+        other = np.setdiff1d(np.arange(2048), read)
+        ram = np.ascontiguousarray(ram)
+        ram[:, :, other] = rng.integers(0, 256, (2 * T, N, len(other)), dtype=np.uint8)
+        frames = rng.choice(np.array([4, 8, 1], np.int32), (2 * T, N))
+        got = {}
+        for dev, lib in libs.items():
+            z = lambda *s, dtype=torch.uint8: torch.zeros(s, dtype=dtype, device=dev)   # noqa: E731
+            st, rd, keys = z(N, 80), z(N, 120), z(max(N * cap, 1), dtype=torch.int32)
+            for half in range(2):
+                buf = z(T * N * 2048 + 1)
+                buf[1:] = torch.from_numpy(ram[half * T:(half + 1) * T].reshape(-1)).to(dev)
+                fr = torch.from_numpy(frames[half * T:(half + 1) * T].copy()).to(dev)
+                out = [z(T, N, dtype=torch.float64), z(T, N), z(T, N, dtype=torch.int32),
+                       z(T, N, dtype=torch.int32), z(T, N, dtype=torch.int32), z(T, N)]
+                s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream if dev == 'cuda' else 0)
+                assert lib.rl10_run(gi, ctypes.c_void_p(buf.data_ptr() + 1), T, N, tptr(fr), tptr(st), tptr(rd),
+                                    tptr(keys), *[tptr(x) for x in out], s) == 0
+                got[dev, half] = [x.cpu().numpy().copy() for x in out + [st, rd, keys]]
+        for half in range(2):
+            for k, (a, b) in enumerate(zip(got['cpu', half], got['cuda', half])):
+                np.testing.assert_array_equal(a, b, err_msg=f'{game}: call {half}, buffer {k}')
