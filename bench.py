@@ -640,13 +640,13 @@ def bench_reward10(args, K, W, baseline):
                kernels=dict(rl10_smb_run=dict(ms_per_launch=round(kms, 4), alg_bytes_per_launch=alg,
                                               achieved_gbps=round(achieved, 3),
                                               clocks_per_step=round(kms * 1e-3 * CLOCK_HZ / T, 1),
-                                              launches='k_smb_signals, k_smb_chain, k_smb_reward')),
+                                              launches='k_smb_run')),
                roofline=dict(kernel='rl10_smb_run', bound='hbm', achieved=round(achieved, 3), peak=HBM_PEAK_GBPS,
                              unit='GB/s', frac=round(achieved / HBM_PEAK_GBPS, 6), traffic=_rl10_traffic(N * T),
                              limiter='issue latency',
-                             note='k_smb_chain, one env per lane for T steps in order, issues one instruction of a '
-                                  'step every 4 cycles (one wave per SIMD on 128 of them); the signals and the '
-                                  'rewards run over all env-steps in parallel'))
+                             note='k_smb_run: the tracker state as two chains, one env per lane, on waves of their own '
+                                  '(the slower issues about 30 instructions a step), the signals and the rewards on '
+                                  'the workgroup\'s other waves'))
     if not args.no_cpu:
         got_r, got_d = rew.cpu().numpy(), done.cpu().numpy()
         lib_o = _oracle()

@@ -337,116 +337,140 @@ __global__ void k_gather_rows(uint4* __restrict__ dst, const uint4* __restrict__
     for (size_t i = blockIdx.y * blockDim.x + threadIdx.x; i < row_vecs; i += (size_t)gridDim.y * blockDim.x) d[i] = s[i];
 }
 
-// Standalone reward10 SMB tracker (smb_tracker.h): the signals and what depends only on them for every env-step in
-// parallel, the tracker state env by env, the rewards in parallel.
-// 1. Four consecutive steps of one env per thread (rows t-1 .. t+3 of ram15 read once).
-__global__ __launch_bounds__(256) void k_smb_signals(const uint8_t* __restrict__ ram15, int T, int N,
-                                                      const Rl10State* __restrict__ state, ev::SmbStep* __restrict__ rec) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const size_t groups = (size_t)((T + 3) / 4) * (size_t)N;
-    if (i >= groups) return;
-    const int e = (int)(i % (size_t)N), t0 = (int)(i / (size_t)N) * 4;
-    const uint4* src = reinterpret_cast<const uint4*>(ram15);
+// Standalone reward10 SMB tracker (smb_tracker.h): waves 0 and 1 of a workgroup run the two chains of its kSmbEnvs
+// envs, one env per lane, the others the passes before and after them, each pass one chunk of kSmbSteps steps behind
+// the one before it, a barrier a chunk.
+// Bound: the slower chain, about 30 instructions a step, one lane in two idle, issued once in 4 cycles or later: 127 us
+// for 8192 envs x 1024 steps, 298 clocks a step (one chain of 79 instructions behind a pass over memory on each side,
+// 16-byte records between them: 290 us, of it 203 us for the chain at 477 clocks a step). 32 envs a workgroup, so that
+// 8192 envs are one workgroup a CU; with the records in LDS the call reads its 16 bytes and writes its 5 an env-step.
+__global__ __launch_bounds__(64 * (2 + ev::kSmbHelpers)) void k_smb_run(const uint4* __restrict__ ram15, int T, int N,
+                                                                       int frames, Rl10State* __restrict__ state,
+                                                                       float* __restrict__ reward,
+                                                                       uint8_t* __restrict__ done) {
+    constexpr int E = ev::kSmbEnvs, K = ev::kSmbSteps;
+    __shared__ uint4 rec[2][K][E];       // pass 1 -> 2
+    __shared__ uint4 dec[3][K][E];       // pass 2 -> 3, 4
+    __shared__ double score[4][K][E];    // pass 1 -> 3 -> 4
+    __shared__ int end_step[E];          // the step that ended the episode; -1: before this call; T: none
+    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+    const int group = (int)((blockIdx.x & 7u) * (gridDim.x >> 3) + (blockIdx.x >> 3));   // (the grid is a multiple of 8)
+    if (group * E >= N) return;
+    const int env = lane % E, e = group * E + env;
+    const bool live = e < N;
     const Rl10Game G = rl10_game(RL10_SMB);
-    auto signals = [&](int t) {
-        const uint4 q = src[(size_t)t * N + e];
-        uint8_t b[16];
-        memcpy(b, &q, 16);
-        return ev::smb_signals(b);
-    };
-    Rl10Signals p;
-    bool had;
-    if (t0 > 0) {
-        p = signals(t0 - 1);
-        had = true;
-    } else {
-        p = state[e].prev;
-        had = state[e].has_prev != 0;
+    const int chunks = (T + K - 1) / K;
+    const Rl10State* saved = &state[live ? e : N - 1];
+    if (wave < 2) {
+        __builtin_amdgcn_s_setprio(3);   // the chains are what the call waits for
+        const int64_t stall = (int64_t)__builtin_ceil(G.stall_frames);
+        ev::SmbLevels lv{saved->has_best_level ? saved->best_level : ev::kSmbNoLevel,
+                         saved->has_best_progress ? (int32_t)saved->best_progress : ev::kSmbNoBest, ev::kSmbNoBest};
+        ev::SmbBudget bu{saved->score_used, saved->idle_frames, saved->deaths};
+        ev::SmbBudget end_bu = bu;       // as the ending step left them
+        uint4 end_dec{(uint32_t)lv.level, (uint32_t)lv.best, (uint32_t)ev::kSmbNoBest, 0u};
+        int ended = saved->done ? -1 : T;
+        if (wave == 1 && lane < E) end_step[env] = ended;
+        for (int i = 0; i < chunks + 3; ++i) {
+            const int c = i - 1 - wave, n = min(K, T - c * K);
+            if (c >= 0 && n > 0 && lane < E) {
+                const uint4* in = &rec[c & 1][0][env];
+                uint4* out = &dec[c % 3][0][env];
+                double* sc = &score[c & 3][0][env];
+                if (wave == 0) {
+                    if (n == K) {
+#pragma unroll
+                        for (int j = 0; j < K; ++j) out[j * E] = lv.step(in[j * E]);
+                    } else {
+                        for (int j = 0; j < n; ++j) out[j * E] = lv.step(in[j * E]);
+                    }
+                } else {
+                    auto step = [&](int j) {
+                        double s = sc[j * E];
+                        const bool ends = bu.step(out[j * E].w, &s, frames, stall);
+                        sc[j * E] = s;
+                        if (ends && ended == T) {   // once an episode: the state is kept as it is now
+                            ended = c * K + j;
+                            end_step[env] = ended;
+                            end_bu = bu;
+                            end_dec = out[j * E];
+                        }
+                    };
+                    if (n == K) {
+#pragma unroll
+                        for (int j = 0; j < K; ++j) step(j);
+                    } else {
+                        for (int j = 0; j < n; ++j) step(j);
+                    }
+                    if (c == chunks - 1 && ended == T) {
+                        end_bu = bu;
+                        end_dec = out[(n - 1) * E];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        if (wave == 1 && lane < E && live) {
+            Rl10State st = *saved;
+            if (ended >= 0) {   // (a tracker that was done before keeps its state)
+                const int32_t level = (int32_t)end_dec.x, last = (int32_t)end_dec.z;
+                const int32_t best = (end_dec.w & ev::DC_BETTER) ? last : (int32_t)end_dec.y;
+                st.has_best_level = level != ev::kSmbNoLevel;
+                if (level != ev::kSmbNoLevel) st.best_level = level;
+                st.has_best_progress = best != ev::kSmbNoBest;
+                if (last != ev::kSmbNoBest) st.best_progress = (double)last;
+                st.deaths = end_bu.deaths;
+                st.idle_frames = end_bu.idle;
+                st.score_used = end_bu.used;
+                if (ended < T) {
+                    st.done = 1;
+                    st.end_reason = (uint8_t)ev::smb_end_reason(end_dec.w);
+                }
+            }
+            const uint4 q = ram15[(size_t)(T - 1) * N + e];   // update's prev: the signals of the last step
+            uint8_t bytes[16];
+            memcpy(bytes, &q, 16);
+            st.has_prev = 1;
+            st.prev = ev::smb_signals(bytes);
+            state[e] = st;
+        }
+        return;
     }
-    for (int k = 0; k < 4 && t0 + k < T; ++k) {
-        const Rl10Signals s = signals(t0 + k);
-        rec[(size_t)(t0 + k) * N + e] = ev::smb_step_record(s, p, had, G);
-        p = s;
-        had = true;
+    // passes 1 and 4: steps 2 j and 2 j + 1 of a chunk, the rows t - 1 .. t + 1 loaded a chunk ahead
+    const int j = ((wave - 2) * 2 + lane / E) * 2;
+    const uint4* src = ram15 + (live ? e : N - 1);
+    auto row = [&](int t) { return src[(size_t)min(max(t, 0), T - 1) * N]; };
+    uint4 q0 = row(j - 1), q1 = row(j), q2 = row(j + 1);
+    const bool had0 = saved->has_prev != 0;
+    const ev::SmbSignals before = ev::smb_saved_signals(saved->prev);
+    for (int i = 0; i < chunks + 3; ++i) {
+        if (i < chunks) {
+            const int t = i * K + j;
+            const ev::SmbSignals p = t > 0 ? ev::smb_step_signals(q0) : before;
+            const ev::SmbSignals s1 = ev::smb_step_signals(q1), s2 = ev::smb_step_signals(q2);
+            q0 = row(t + K - 1);
+            q1 = row(t + K);
+            q2 = row(t + K + 1);
+            rec[i & 1][j][env] = ev::smb_step(s1, p, t > 0 || had0, G, &score[i & 3][j][env]);
+            rec[i & 1][j + 1][env] = ev::smb_step(s2, s1, true, G, &score[i & 3][j + 1][env]);
+        }
+        const int c = i - 3;
+        if (c >= 0 && live) {
+            const int ended = end_step[env];
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                const int t = c * K + j + k;
+                if (t < T) {
+                    const size_t at = (size_t)t * N + e;
+                    const double r = ev::smb_reward(dec[c % 3][j + k][env], score[c & 3][j + k][env], t == ended,
+                                                    frames, G);
+                    reward[at] = t <= ended ? (float)r : 0.0f;
+                    done[at] = t >= ended ? 1 : 0;
+                }
+            }
+        }
+        __syncthreads();
     }
-}
-// 2. One env per lane (64-lane blocks: as many CUs as waves), its steps in order; the records of kAhead steps are
-// loaded ahead in two register buffers, through row bases that are the same for the whole wave (the buffer holds
-// kAhead rows past the last, which the last loads read and nothing uses).
-constexpr int kAhead = 4;
-__global__ __launch_bounds__(64) void k_smb_chain(ev::SmbStep* __restrict__ rec, const uint8_t* __restrict__ ram15,
-                                                   int T, int N, int frames, Rl10State* __restrict__ state) {
-    const int e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (e >= N) return;
-    const Rl10Game G = rl10_game(RL10_SMB);
-    const int64_t stall = G.stall_frames >= 0.0 ? (int64_t)__builtin_ceil(G.stall_frames) : -1;
-    auto row = [&](int t) { return rec + (size_t)(uint32_t)t * (uint32_t)N; };
-    auto put = [&](int t, const ev::SmbDec& d) { reinterpret_cast<ev::SmbDec*>(row(t))[e] = d; };
-    Rl10State st = state[e];
-    ev::SmbChain c{st.done ? 1u : 0u, 0u, st.has_best_level ? st.best_level : -1,
-                   st.has_best_progress ? (int32_t)st.best_progress : ev::kNoBest, ev::kNoBest, st.deaths,
-                   st.idle_frames, st.score_used};
-    ev::SmbStep a[kAhead], b[kAhead];
-#pragma unroll
-    for (int j = 0; j < kAhead; ++j) a[j] = row(j)[e];
-    int t = 0;
-    for (; t + 2 * kAhead <= T; t += 2 * kAhead) {
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) b[j] = row(t + kAhead + j)[e];
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) put(t + j, ev::smb_chain_step(a[j], frames, c, stall));
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) a[j] = row(t + 2 * kAhead + j)[e];
-#pragma unroll
-        for (int j = 0; j < kAhead; ++j) put(t + kAhead + j, ev::smb_chain_step(b[j], frames, c, stall));
-    }
-    for (; t < T; ++t) put(t, ev::smb_chain_step(row(t)[e], frames, c, stall));   // the last T % 8 steps
-    st.done = (uint8_t)c.done;
-    if (c.end_flags) st.end_reason = (uint8_t)ev::smb_end_reason(c.end_flags);   // ended in this call
-    st.has_best_level = c.best_level >= 0 ? 1 : 0;
-    if (c.best_level >= 0) st.best_level = c.best_level;
-    st.has_best_progress = c.best_progress != ev::kNoBest ? 1 : 0;
-    if (c.last_progress != ev::kNoBest) st.best_progress = (double)c.last_progress;
-    st.deaths = c.deaths;
-    st.idle_frames = c.idle;
-    st.score_used = c.score_used;
-    if (T > 0) {   // update's prev: the signals of the last step
-        const uint4 q = reinterpret_cast<const uint4*>(ram15)[(size_t)(T - 1) * N + e];
-        uint8_t bb[16];
-        memcpy(bb, &q, 16);
-        st.has_prev = 1;
-        st.prev = ev::smb_signals(bb);
-    }
-    state[e] = st;
-}
-// 3. The rewards and done flags of every env-step.
-__global__ __launch_bounds__(256) void k_smb_reward(const ev::SmbDec* __restrict__ dec, size_t n, int frames,
-                                                     float* __restrict__ reward, uint8_t* __restrict__ done) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= n) return;
-    const ev::SmbDec d = dec[i];
-    reward[i] = (float)ev::smb_reward(d, frames, rl10_game(RL10_SMB));
-    done[i] = (d.flags & ev::DC_DONE) ? 1 : 0;
-}
-
-// The per-step records of rl10_smb_run come from a stream-ordered pool of the device (allocated and freed on the
-// caller's stream, so calls on different streams never share one), which keeps its memory for the next call.
-hipMemPool_t smb_pool(int device) {
-    static std::mutex lock;
-    static std::map<int, hipMemPool_t> pools;
-    std::lock_guard<std::mutex> hold(lock);
-    auto it = pools.find(device);
-    if (it != pools.end()) return it->second;
-    hipMemPoolProps props{};
-    props.allocType = hipMemAllocationTypePinned;
-    props.location.type = hipMemLocationTypeDevice;
-    props.location.id = device;
-    hipMemPool_t pool = nullptr;
-    if (hipMemPoolCreate(&pool, &props) != hipSuccess) throw std::runtime_error("hipMemPoolCreate failed");
-    uint64_t keep = ~0ull;
-    (void)hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &keep);
-    pools.emplace(device, pool);
-    return pool;
 }
 
 // Standalone reward10 tracker of any game, T steps over the 2 KB RAM of each env-step.
@@ -1929,29 +1953,11 @@ int rl_stream_destroy(void* stream) {
 int rl10_smb_run(const uint8_t* ram15, int T, int N, int frames, void* state, float* reward, uint8_t* done,
                  void* stream) {
     if (N <= 0 || T <= 0) return check("rl10_smb_run");
-    try {
-        const hipStream_t st = static_cast<hipStream_t>(stream);
-        int device = 0;
-        if (hipGetDevice(&device) != hipSuccess) throw std::runtime_error("hipGetDevice failed");
-        const size_t n = (size_t)T * (size_t)N;
-        void* rec = nullptr;   // (kAhead rows past the last: k_smb_chain's last loads)
-        if (hipMallocFromPoolAsync(&rec, (n + (size_t)kAhead * (size_t)N) * sizeof(ev::SmbStep), smb_pool(device), st) !=
-            hipSuccess)
-            throw std::runtime_error("rl10_smb_run: no device memory for the per-step records");
-        const size_t groups = (size_t)((T + 3) / 4) * (size_t)N;
-        hipLaunchKernelGGL(k_smb_signals, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, st, ram15, T, N,
-                           static_cast<const Rl10State*>(state), static_cast<ev::SmbStep*>(rec));
-        hipLaunchKernelGGL(k_smb_chain, dim3((N + 63) / 64), dim3(64), 0, st, static_cast<ev::SmbStep*>(rec), ram15, T,
-                           N, frames, static_cast<Rl10State*>(state));
-        hipLaunchKernelGGL(k_smb_reward, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st,
-                           static_cast<const ev::SmbDec*>(rec), n, frames, reward, done);
-        const int bad = check("rl10_smb_run");
-        (void)hipFreeAsync(rec, st);
-        return bad;
-    } catch (const std::exception& ex) {
-        g_error = ex.what();
-        return 1;
-    }
+    const unsigned groups = ((unsigned)N + ev::kSmbEnvs - 1) / ev::kSmbEnvs;
+    hipLaunchKernelGGL(k_smb_run, dim3((groups + 7) / 8 * 8), dim3(64 * (2 + ev::kSmbHelpers)), 0,
+                       static_cast<hipStream_t>(stream), reinterpret_cast<const uint4*>(ram15), T, N, frames,
+                       static_cast<Rl10State*>(state), reward, done);
+    return check("rl10_smb_run");
 }
 
 int rl10_run(int game, const uint8_t* ram, int T, int N, const int32_t* frames, void* state, void* reader,

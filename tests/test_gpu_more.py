@@ -242,3 +242,30 @@ def test_reward10_kernel_every_path_over_split_calls():
         t0 += n_steps
     ends = st_c.reshape(N, 80)[:, 4]          # Rl10State.end_reason
     assert set(np.unique(ends).tolist()) >= {1, 2, 3, 4}, np.unique(ends, return_counts=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('T,N', [(1, 1), (23, 31), (24, 32), (25, 33), (47, 64), (73, 257)])
+def test_reward10_kernel_chunk_and_group_edges(T, N):
+    """rl10_smb_run at the edges of its chunks of 24 steps and groups of 32 envs, three calls in a row on trajectories
+    that reach every end: rewards, done flags and tracker state equal the oracle's."""
+    print(f'case: rl10_smb_run, three calls of T={T} N={N}, every tracker path', flush=True)
+    lib = ctypes.CDLL(str(HIP_LIB))
+    lib.rl10_smb_run.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
+                                 ctypes.c_void_p, ctypes.c_void_p, ctypes.c_void_p]
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    ram = stress_ram15(T, N, 3 * T, level_up_at=T - 1)
+    st_c = np.zeros(N * 80, np.uint8)
+    st_g = torch.zeros(N * 80, dtype=torch.uint8, device='cuda')
+    for c, frames in enumerate((4, 300, 4)):
+        part = np.ascontiguousarray(ram[c * T:(c + 1) * T])
+        want_r, want_d = np.zeros((T, N), np.float32), np.zeros((T, N), np.uint8)
+        assert oracle().rl10_smb_run(ptr(part), T, N, frames, ptr(st_c), ptr(want_r), ptr(want_d), None) == 0
+        rew = torch.zeros(T, N, dtype=torch.float32, device='cuda')
+        done = torch.zeros(T, N, dtype=torch.uint8, device='cuda')
+        assert lib.rl10_smb_run(tptr(torch.from_numpy(part).cuda()), T, N, frames, tptr(st_g), tptr(rew), tptr(done),
+                                s) == 0
+        torch.cuda.synchronize()
+        assert np.array_equal(rew.cpu().numpy(), want_r), c
+        assert np.array_equal(done.cpu().numpy(), want_d), c
+        assert np.array_equal(st_g.cpu().numpy(), st_c), c
