@@ -3,6 +3,7 @@
 pass of k_emu_w), weighted plans over places, and the start/level/progress outputs; the archive is compared through
 the exact-resume blob."""
 import ctypes
+import os
 
 import numpy as np
 import pytest
@@ -145,4 +146,32 @@ def test_grown_archive_resumes_on_both_builds():
             assert np.array_equal(getattr(cpu, k).numpy(), getattr(gpu, k).cpu().numpy()), (t, k)
         starts += int(((cpu.start_level >= 0) & (cpu.done > 0)).sum())
     assert starts > 0
+    assert np.array_equal(cpu.state_dict()['env'], gpu.state_dict()['env'])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('idle,n', [(0, 12), (3, 12), (9, 65)])
+def test_translated_level_starts(idle, n):
+    """A level start's idle and restart frames on the translated kernel (RLENV_JIT=sync), with no idle frames (its
+    idle pass is not launched) and with more consoles than a wave has lanes."""
+    print(f'case: SMB-like cart seed 2 translated, {n} consoles, level_cap 4, idle 0..{idle}, 110 decisions, then '
+          'p(level start) 0.7 with Geometric(1/5) ends for 16 decisions', flush=True)
+    os.environ['RLENV_JIT'] = 'sync'
+    try:
+        cpu, gpu = pair(n, seed=32, sticky=True, idle_max=idle, dropout=True, pad_mode=True, level_cap=4)
+    finally:
+        del os.environ['RLENV_JIT']
+    assert gpu.jit_status(0)['state'] == 'loaded'
+    g = torch.Generator().manual_seed(5)
+    cpu.start()
+    gpu.start()
+    run_pair(cpu, gpu, 0, 110, g, check_every=55)
+    for e in (cpu, gpu):
+        e.set_level_prob(0.7)
+        set_end(e, 1 / 5)
+    starts = 0
+    for t in range(110, 126):
+        run_pair(cpu, gpu, t, 1, g)
+        starts += int((cpu.start_level.numpy() >= 0).sum())
+    assert starts > 0, 'no finished episode had started from a level start'
     assert np.array_equal(cpu.state_dict()['env'], gpu.state_dict()['env'])
