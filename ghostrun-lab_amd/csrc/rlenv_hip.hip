@@ -340,10 +340,11 @@ __global__ void k_gather_rows(uint4* __restrict__ dst, const uint4* __restrict__
 // Standalone reward10 SMB tracker (smb_tracker.h): waves 0 and 1 of a workgroup run the two chains of its kSmbEnvs
 // envs, one env per lane, the others the passes before and after them, each pass one chunk of kSmbSteps steps behind
 // the one before it, a barrier a chunk.
-// Bound: the slower chain, about 30 instructions a step, one lane in two idle, issued once in 4 cycles or later: 127 us
-// for 8192 envs x 1024 steps, 298 clocks a step (one chain of 79 instructions behind a pass over memory on each side,
-// 16-byte records between them: 290 us, of it 203 us for the chain at 477 clocks a step). 32 envs a workgroup, so that
-// 8192 envs are one workgroup a CU; with the records in LDS the call reads its 16 bytes and writes its 5 an env-step.
+// Bound: the chains, 26 and 28 instructions a step, each issued once in 4 cycles or later: 101 us for 8192 envs x 1024
+// steps, 236 clocks a step (127 us with a branch on the end after each step of the second chain, which waited for the
+// step's inputs in LDS; 290 us as one chain of 79 instructions a step, 477 clocks, behind a pass over memory on each
+// side with 16-byte records between them). 32 envs a workgroup, so that 8192 envs are one workgroup a CU; with the
+// records in LDS the call reads its 16 bytes and writes its 5 an env-step.
 __global__ __launch_bounds__(64 * (2 + ev::kSmbHelpers)) void k_smb_run(const uint4* __restrict__ ram15, int T, int N,
                                                                        int frames, Rl10State* __restrict__ state,
                                                                        float* __restrict__ reward,
@@ -385,22 +386,31 @@ __global__ __launch_bounds__(64 * (2 + ev::kSmbHelpers)) void k_smb_run(const ui
                         for (int j = 0; j < n; ++j) out[j * E] = lv.step(in[j * E]);
                     }
                 } else {
-                    auto step = [&](int j) {
-                        double s = sc[j * E];
-                        const bool ends = bu.step(out[j * E].w, &s, frames, stall);
-                        sc[j * E] = s;
-                        if (ends && ended == T) {   // once an episode: the state is kept as it is now
-                            ended = c * K + j;
-                            end_step[env] = ended;
-                            end_bu = bu;
-                            end_dec = out[j * E];
-                        }
-                    };
-                    if (n == K) {
+                    const ev::SmbBudget from = bu;
+                    bool ends = false;
+                    if (n == K) {   // (the chunk's inputs loaded at once, and no branch between its steps)
+                        uint32_t f[K];
+                        double s[K];
 #pragma unroll
-                        for (int j = 0; j < K; ++j) step(j);
+                        for (int j = 0; j < K; ++j) {
+                            f[j] = out[j * E].w;
+                            s[j] = sc[j * E];
+                        }
+#pragma unroll
+                        for (int j = 0; j < K; ++j) {
+                            ends |= bu.step(f[j], &s[j], frames, stall);
+                            sc[j * E] = s[j];
+                        }
                     } else {
-                        for (int j = 0; j < n; ++j) step(j);
+                        for (int j = 0; j < n; ++j) ends |= bu.step(out[j * E].w, &sc[j * E], frames, stall);
+                    }
+                    if (ends && ended == T) {   // once an episode: the chunk again (the terms give themselves), up to
+                        end_bu = from;          // the step that ends it, for the state as it leaves it
+                        int j = 0;
+                        for (double s = sc[0]; !end_bu.step(out[j * E].w, &s, frames, stall); s = sc[j * E]) ++j;
+                        ended = c * K + j;
+                        end_step[env] = ended;
+                        end_dec = out[j * E];
                     }
                     if (c == chunks - 1 && ended == T) {
                         end_bu = bu;
