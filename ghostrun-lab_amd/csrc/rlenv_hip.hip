@@ -1195,22 +1195,25 @@ void restart_phases(const Env& env, const GameK& g, const Outs& o, int e0, int e
 
 // A decision of envs [e0, e1) of game g: 4 frames, then the finish, the level saves and the restart pass.
 // Pipelined (a one-game env whose frame launch fits in one round of waves, so that waves retiring from the
-// emulator leave CU slots idle): frames 0 and 1 are drawn on the game's render stream from frame banks 0 and 1 while
-// the frames after them are emulated on `st`, frames 2 and 3 by the waves that emulate them (drawn on the render
-// stream too, frame 2 left the render stream's last launch running alone after the emulation: 3.42 against 3.33
-// ms per decision of 8192 consoles), and the restart pass, which writes the pictures of restarted envs, waits until
+// emulator leave CU slots idle): the first frames are drawn on the game's render stream from frame banks while the frames
+// after them are emulated on `st`, the others by the waves that emulate them. Up to three quarters of a round frames
+// 0, 1 and 2: a frame's emulation is a chain that the draw, 0.1 ms, would only lengthen (2048 consoles: 1.210 ms a
+// decision against 1.325 with frame 2 drawn in its own waves, 6144: 2.096 against 2.171). Above that frames 0 and 1:
+// the launches fill the GPU, and frame 2's draw left the render stream running alone after the emulation (8192: 2.686
+// against 2.633). The restart pass, which writes the pictures of restarted envs, waits until
 // every frame is drawn (so does the next decision, which refills the banks, through it). Otherwise each frame is
 // drawn on `st` after it is emulated: with several rounds of waves, or with other games' streams, the CUs are
 // already kept busy.
-constexpr int kBankFrames = 2;   // decision frames drawn on the render stream when pipelined: 0 .. kBankFrames - 1
+constexpr int kBankFrames = 3;   // the most decision frames drawn on the render stream, from banks 0 .. kBankFrames - 1
 void decision_phases(const Env& env, const GameK& g, const RenderPipe& p, const Outs& o, int e0, int e1,
                      hipStream_t st) {
     const int n = e1 - e0;
     if (n <= 0) return;
     const bool draw = !env.s.no_render;
     const bool pipelined = draw && env.games.size() == 1 && n <= env.one_round;
+    const int banked = 4 * n <= 3 * env.one_round ? kBankFrames : kBankFrames - 1;
     for (int f = 0; f < RLE_FRAMES; ++f) {
-        if (!pipelined || f >= kBankFrames) {   // emulated and drawn by the same waves; the last one finishes too
+        if (!pipelined || f >= banked) {   // emulated and drawn by the same waves; the last one finishes too
             launch_emu(env, g, o, EMU_DECISION, f, false, e0, e1, st, -1, true, f == RLE_FRAMES - 1);
             continue;
         }
