@@ -803,9 +803,13 @@ void jit_enqueue(const std::shared_ptr<JitJob>& job) {
     q.cv.notify_all();
 }
 
-// The job of (blocks, source): this process's existing one (fresh = false), or a new one the caller compiles.
-constexpr int kJitMinEnvs = 1024;   // games of fewer envs run the library's kernel unless RLENV_JIT=sync
+// Games of fewer envs run the library's kernel unless RLENV_JIT=sync. A decision of a small game is a chain of four
+// frames whatever its size, and the translated chain is 4 to 5 times as short (500 NROM consoles: 5.36 against 1.08 ms a
+// decision), so the line is the compile's cost against the decisions of a run, not a size where one kernel passes the
+// other: a fixed-PRG cart compiles in 15 to 35 s, a banked one in four times that, for four times the envs.
+constexpr int kJitMinEnvsFixed = 256, kJitMinEnvsBanked = 1024;
 
+// The job of (blocks, source): this process's existing one (fresh = false), or a new one the caller compiles.
 std::shared_ptr<JitJob> jit_job(std::string blocks, std::string source, bool& fresh) {
     static std::mutex lock;
     static std::map<std::string, std::shared_ptr<JitJob>> jobs;
@@ -1406,9 +1410,8 @@ void* rlenv_create(int ngames, const int* game_ids, const uint8_t* const* roms, 
         e.ep_maxlvl = env->mem.zeros<int32_t>(N);
         e.ep_idle = env->mem.zeros<int32_t>(N);
         e.resetting = env->mem.zeros<uint8_t>(N);
-        // translated kernels (jit.h): by default every game of at least kJitMinEnvs envs (a smaller one gains less
-        // than the compile takes), compiled in the background; RLENV_JIT=fixed: only the fixed-PRG games of that
-        // size (a banked cart's translation is larger, tens of seconds of compile); sync: every game, compiled
+        // translated kernels (jit.h): by default every game of at least kJitMinEnvsFixed or kJitMinEnvsBanked envs,
+        // compiled in the background; RLENV_JIT=fixed: only the fixed-PRG games of that size; sync: every game, compiled
         // before rlenv_create returns; 0 (or off): none
         const char* jv = std::getenv("RLENV_JIT");
         const int jit_mode = !jv ? 2 : (!strcmp(jv, "0") || !strcmp(jv, "off")) ? 0 : !strcmp(jv, "sync") ? 3
@@ -1489,7 +1492,8 @@ void* rlenv_create(int ngames, const int* game_ids, const uint8_t* const* roms, 
                 }
             }
             // the translation, and a fetch table with its blocks' keys (by CPU address, or by PRG offset)
-            if (jit_mode == 3 || (jit_mode >= 1 && g.n >= kJitMinEnvs && (fixed32 || jit_mode == 2))) {
+            if (jit_mode == 3 || (fixed32 ? jit_mode >= 1 && g.n >= kJitMinEnvsFixed
+                                          : jit_mode == 2 && g.n >= kJitMinEnvsBanked)) {
                 JitProgram jp = fixed32 ? jit_translate_fixed(img) : jit_translate_banked(p.prg, p.board);
                 if (!jp.leader_addr.empty()) {
                     std::vector<uint32_t> fj(f);

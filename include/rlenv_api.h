@@ -116,8 +116,8 @@ int rlenv_kernel_times(void* h, double* ms, int64_t* count, int n);
  * cart's 6502 code into blocks of the interpreter's per-opcode handlers with constant operands (by CPU address on
  * NROM and CNROM, by PRG offset on the banked boards) and compiles them at run time (hiprtc; the games' compiles in
  * parallel, each translation once per process) into a copy of the console-frame kernel that the game's decision
- * frames then use; a console's results are the same on either kernel. Which games: by default every game of at least
- * 1024 envs; RLENV_JIT=fixed: only the fixed-PRG games of that size; RLENV_JIT=sync: every game; RLENV_JIT=0 (or off):
+ * frames then use; a console's results are the same on either kernel. Which games: by default every fixed-PRG game (NROM,
+ * CNROM) of at least 256 envs and every other of at least 1024; RLENV_JIT=fixed: only the fixed-PRG games of that size; RLENV_JIT=sync: every game; RLENV_JIT=0 (or off):
  * none. The compiles run on one thread of the process, one at a time, in the order asked for, while rlenv_create
  * returns at once (RLENV_JIT=sync: after them); a game's decision frames switch to its translated kernel at the first
  * rlenv_step, rlenv_step_game, rlenv_step_range, rlenv_jit_wait or rlenv_jit_status after its compile (never in the
