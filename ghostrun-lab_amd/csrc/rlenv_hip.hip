@@ -340,11 +340,12 @@ __global__ void k_gather_rows(uint4* __restrict__ dst, const uint4* __restrict__
 // Standalone reward10 SMB tracker (smb_tracker.h): waves 0 and 1 of a workgroup run the two chains of its kSmbEnvs
 // envs, one env per lane, the others the passes before and after them, each pass one chunk of kSmbSteps steps behind
 // the one before it, a barrier a chunk.
-// Bound: the chains, 26 and 28 instructions a step, each issued once in 4 cycles or later: 101 us for 8192 envs x 1024
-// steps, 236 clocks a step (127 us with a branch on the end after each step of the second chain, which waited for the
-// step's inputs in LDS; 290 us as one chain of 79 instructions a step, 477 clocks, behind a pass over memory on each
-// side with 16-byte records between them). 32 envs a workgroup, so that 8192 envs are one workgroup a CU; with the
-// records in LDS the call reads its 16 bytes and writes its 5 an env-step.
+// Bound: the chains, 30 and 23 instructions a step, each issued once in 4 cycles or later: 97 us for 8192 envs x 1024
+// steps, 227 clocks a step (101 us with a subtraction and an "and" more between a step's level and the next one's; 127
+// us with a branch on the end after each step of the second chain, which waited for the step's inputs in LDS; 290 us
+// as one chain of 79 instructions a step, 477 clocks, behind a pass over memory on each side with 16-byte records
+// between them). 32 envs a workgroup, so that 8192 envs are one workgroup a CU; with the records in LDS the call reads
+// its 16 bytes and writes its 5 an env-step.
 __global__ __launch_bounds__(64 * (2 + ev::kSmbHelpers)) void k_smb_run(const uint4* __restrict__ ram15, int T, int N,
                                                                        int frames, Rl10State* __restrict__ state,
                                                                        float* __restrict__ reward,

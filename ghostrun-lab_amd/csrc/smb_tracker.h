@@ -98,17 +98,17 @@ struct SmbLevels {
     int32_t level, best, last;
     __device__ __forceinline__ uint4 step(const uint4& q) {
         const int32_t at = (int32_t)q.x, progress = (int32_t)q.y;
-        const int32_t d = at - level;
-        const bool up = d == 1, skip = d > 1;
-        const bool first = (uint32_t)(d + kSmbNoLevel) < 0x10000u;   // in play and no best level yet
+        // (the next step waits for level and best only: a compare and a select, a select and a maximum)
+        const bool up = at - 1 == level, skip = at - 1 > level;
+        const bool first = level == kSmbNoLevel && at >= 0;          // in play and no best level yet
         const bool reset = up || first;
         level = reset ? at : level;
-        best = reset ? kSmbNoBest : best;
-        const int32_t before = best;
+        const int32_t before = reset ? kSmbNoBest : best;
         const bool at_best = at == level;
-        const bool better = at_best && progress > before;            // a first setting or a gain
+        const int32_t reached = at_best ? progress : kSmbNoBest;
+        const bool better = reached > before;                        // a first setting or a gain
         const bool gain = better && before != kSmbNoBest;
-        best = better ? progress : before;
+        best = reached > before ? reached : before;
         last = better ? progress : last;
         const uint32_t f = q.z | (up ? DC_LEVEL : 0u) | (gain ? DC_GAIN : 0u) | (skip ? DC_SKIP : 0u) |
                            (at_best ? DC_AT_BEST : 0u) | (better ? DC_BETTER : 0u) | (reset ? DC_RESET : 0u);
@@ -125,8 +125,8 @@ struct SmbBudget {
     int32_t deaths;
     __device__ __forceinline__ bool step(uint32_t f, double* score, int frames, int64_t stall) {
         used = (f & DC_RESET) ? 0.0 : used;
-        const double left = kScoreBudget - used, sr = left < *score ? left : *score;
-        used += sr > 0.0 ? sr : 0.0;
+        const double sr = __builtin_fmin(kScoreBudget - used, *score);   // (both finite)
+        used += __builtin_fmax(sr, 0.0);
         *score = sr;
         deaths += (int32_t)((f >> 4) & 1u);   // ST_DEATH
         const int64_t more = idle + frames;
