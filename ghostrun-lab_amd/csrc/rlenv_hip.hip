@@ -1132,7 +1132,7 @@ void launch_emu(const Env& env, const GameK& g, const Outs& o, int mode, int f, 
     // level start, 16.1 ms with those frames on the interpreter.
     JitSlot* js = blocks > 0 ? jit_slot(env, g) : nullptr;
     hipFunction_t fn = nullptr;
-    if (js && js->fn_draw) fn = draw || mode != EMU_DECISION ? js->fn_draw : a.bank ? js->fn : nullptr;
+    if (js && js->fn_draw) fn = a.bank ? js->fn : draw || mode != EMU_DECISION ? js->fn_draw : nullptr;
     if (fn) {
         a.g.cart.fetchw = js->fetchw;
         void* args[] = {&a};
@@ -1174,8 +1174,12 @@ void launch_render(const Env& env, const GameK& g, const Outs& o, int f, bool us
     trace(restart ? "render_restart" : "render", st);
 }
 
+constexpr int kBankFrames = 3;   // the most frames drawn on the render stream, from banks 0 .. kBankFrames - 1
+
 // The restart half of a decision / start: snapshot copy, 4 neutral frames with pictures, first tracker update.
-void restart_phases(const Env& env, const GameK& g, const Outs& o, int e0, int e1, hipStream_t st) {
+// p: the render stream, idle, with the frame banks (a pipelined decision), nullptr to draw on `st`.
+void restart_phases(const Env& env, const GameK& g, const Outs& o, int e0, int e1, hipStream_t st,
+                    const RenderPipe* p = nullptr) {
     const FinishArgs fa = finish_args(env, g, e0, e1, o);
     const int n = e1 - e0;
     env.clock.run(KC_RESET_COPY, st, [&] {
@@ -1187,9 +1191,22 @@ void restart_phases(const Env& env, const GameK& g, const Outs& o, int e0, int e
     // Only a restart from a saved level start emulates; one from the boot snapshot was a copy.
     if (g.lv.cap > 0) {
         if (env.s.idle_max > 0) launch_emu(env, g, o, EMU_IDLE, 0, true, e0, e1, st);
+        // all but the last restart frame drawn on the render stream while the next ones are emulated, as a decision's
+        // frames are (4096 consoles, restarts from level starts: @@ ms a decision, with the draws on `st` @@)
         for (int f = 0; f < RLE_FRAMES; ++f) {
-            launch_emu(env, g, o, EMU_RESTART, f, true, e0, e1, st);
-            launch_render(env, g, o, f, true, true, e0, e1, st);
+            if (!p || f >= kBankFrames) {
+                launch_emu(env, g, o, EMU_RESTART, f, true, e0, e1, st);
+                launch_render(env, g, o, f, true, true, e0, e1, st);
+                continue;
+            }
+            launch_emu(env, g, o, EMU_RESTART, f, true, e0, e1, st, f);
+            (void)hipEventRecord(p->emulated[f], st);
+            (void)hipStreamWaitEvent(p->stream, p->emulated[f], 0);
+            launch_render(env, g, o, f, true, true, e0, e1, p->stream, f);
+        }
+        if (p) {
+            (void)hipEventRecord(p->drawn, p->stream);
+            (void)hipStreamWaitEvent(st, p->drawn, 0);
         }
     }
     env.clock.run(KC_RESET_FINISH, st,
@@ -1209,7 +1226,6 @@ void restart_phases(const Env& env, const GameK& g, const Outs& o, int e0, int e
 // every frame is drawn (so does the next decision, which refills the banks, through it). Otherwise each frame is
 // drawn on `st` after it is emulated: with several rounds of waves, or with other games' streams, the CUs are
 // already kept busy.
-constexpr int kBankFrames = 3;   // the most decision frames drawn on the render stream, from banks 0 .. kBankFrames - 1
 void decision_phases(const Env& env, const GameK& g, const RenderPipe& p, const Outs& o, int e0, int e1,
                      hipStream_t st) {
     const int n = e1 - e0;
@@ -1235,7 +1251,7 @@ void decision_phases(const Env& env, const GameK& g, const RenderPipe& p, const 
         trace("archive", st);
     }
     if (pipelined) (void)hipStreamWaitEvent(st, p.drawn, 0);
-    restart_phases(env, g, o, e0, e1, st);
+    restart_phases(env, g, o, e0, e1, st, pipelined && g.n <= env.one_round ? &p : nullptr);
 }
 
 // Fetch-table entry of the instruction at a (NROM: a CPU address; banked boards: a PRG byte offset, whose low 13
