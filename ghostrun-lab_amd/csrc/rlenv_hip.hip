@@ -1192,7 +1192,7 @@ void restart_phases(const Env& env, const GameK& g, const Outs& o, int e0, int e
     if (g.lv.cap > 0) {
         if (env.s.idle_max > 0) launch_emu(env, g, o, EMU_IDLE, 0, true, e0, e1, st);
         // all but the last restart frame drawn on the render stream while the next ones are emulated, as a decision's
-        // frames are (4096 consoles, restarts from level starts: @@ ms a decision, with the draws on `st` @@)
+        // frames are (4096 consoles, restarts from level starts: 10.24 ms a decision, with the draws on `st` 10.55)
         for (int f = 0; f < RLE_FRAMES; ++f) {
             if (!p || f >= kBankFrames) {
                 launch_emu(env, g, o, EMU_RESTART, f, true, e0, e1, st);
